@@ -1997,17 +1997,23 @@ __device__ __forceinline__ Acc3 target_walk(const SegDesc& s, uint32_t k0, uint3
     const uint32_t sum = live & (node ? acc : ~self);
     const uint32_t open = node ? live & ~acc : 0u;
     if (COUNT) n_int += (uint32_t)__popc(sum & counted);
+    // Branches, not a weight of 0: a node or leaf that a target does not take may lie at a NaN
+    // or infinity (a massless body there, and every com above it). They cost nothing: a set
+    // whose lanes all pass skips the term (16,384 bodies 57.4 us with zero weights, 56.6 so,
+    // 61.2 with the differences zeroed too; 2^18-body collision 10.2, 9.7, 10.7 ms).
 #pragma unroll
     for (int t = 0; t < kTargets; ++t) {
-      const float r2 = d2[t] + eps2;
-      const float ir = rsqrtf(r2);
-      const float w = (sum >> t) & 1u ? A.w * ir * ir * ir : 0.0f;
-      if (KAHAN) {
-        acc_add<true>(a[t], dx[t] * w, dy[t] * w, dz[t] * w);
-      } else {
-        a[t].x = fmaf(dx[t], w, a[t].x);
-        a[t].y = fmaf(dy[t], w, a[t].y);
-        a[t].z = fmaf(dz[t], w, a[t].z);
+      if ((sum >> t) & 1u) {
+        const float r2 = d2[t] + eps2;
+        const float ir = rsqrtf(r2);
+        const float w = A.w * ir * ir * ir;
+        if (KAHAN) {
+          acc_add<true>(a[t], dx[t] * w, dy[t] * w, dz[t] * w);
+        } else {
+          a[t].x = fmaf(dx[t], w, a[t].x);
+          a[t].y = fmaf(dy[t], w, a[t].y);
+          a[t].z = fmaf(dz[t], w, a[t].z);
+        }
       }
     }
     const unsigned long long mo = __ballot(open != 0u);
