@@ -1326,18 +1326,20 @@ __device__ __forceinline__ void store_node(const SegDesc& s, uint32_t j, const A
   NodeBox bx;
   bx.lo = make_float4(r.mn.x, r.mn.y, r.mn.z, __uint_as_float(lo));
   bx.hi = make_float4(r.mx.x, r.mx.y, r.mx.z, __uint_as_float(hi));
+  // the farthest that a point of the box lies from the com, per axis; without quadrupoles the
+  // square of that distance, summed as the per-target walk sums a target's
+  const float ex = fmaxf(r.com.x - r.mn.x, r.mx.x - r.com.x),
+              ey = fmaxf(r.com.y - r.mn.y, r.mx.y - r.com.y),
+              ez = fmaxf(r.com.z - r.mn.z, r.mx.z - r.com.z);
   if (QUAD) {
     // the group walk's classifier radii: squared monopole-band radius (s / (theta
     // mono_ratio) + delta; FLT_MAX when the band is off) and the node's radius about its
     // com (far-field test)
-    const float ex = fmaxf(r.com.x - r.mn.x, r.mx.x - r.com.x),
-                ey = fmaxf(r.com.y - r.mn.y, r.mx.y - r.com.y),
-                ez = fmaxf(r.com.z - r.mn.z, r.mx.z - r.com.z);
     const float rn = sqrtf(fmaf(ex, ex, fmaf(ey, ey, ez * ez)));
     const float rm = fmaf(size, s.mono_inv, delta);
     nd.h = make_float4(rcrit * rcrit, ch, s.mono_inv > 0.f ? rm * rm : 3.4e38f, rn);
   } else {
-    nd.h = make_float4(rcrit * rcrit, ch, 0.f, 0.f);
+    nd.h = make_float4(rcrit * rcrit, ch, ex * ex + ey * ey + ez * ez, 0.f);
   }
   const size_t j2 = 2 * (size_t)j;
   gstore4(reinterpret_cast<float4*>(s.node), j2, nd.a);
@@ -1931,7 +1933,7 @@ constexpr int kTargetLanes = 64 / kTargets;  // lanes that end with one target's
 // first, which adds at most one entry per level (trees are at most 96 levels deep).
 constexpr uint32_t kOpenCap = 512, kOpenWide = kOpenCap - 160;
 
-template <bool KAHAN, bool COUNT>
+template <bool KAHAN, bool COUNT, bool QUAD>
 __device__ __forceinline__ Acc3 target_walk(const SegDesc& s, uint32_t k0, uint32_t cnt,
                                             bool boxes, uint32_t lane, uint32_t* words,
                                             uint8_t* masks, uint32_t counted,
@@ -1950,7 +1952,6 @@ __device__ __forceinline__ Acc3 target_walk(const SegDesc& s, uint32_t k0, uint3
     mz[t] = lf[4 * q + 2];
     a[t] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   }
-  const bool loose_theta = __float_as_uint(s.theta) > __float_as_uint(1.0f);
   const uint64_t leaf_base = (uint64_t)s.leaf, node_base = (uint64_t)s.node;
   uint32_t sp = 0, u = n == 1 ? 0u : kEntryNode, mk = lane == 0 ? (1u << cnt) - 1u : 0u;
   // every node is pushed at most once; the bound only guards corrupted trees
@@ -1964,11 +1965,13 @@ __device__ __forceinline__ Acc3 target_walk(const SegDesc& s, uint32_t k0, uint3
     float d2[kTargets], dx[kTargets], dy[kTargets], dz[kTargets];
     uint32_t acc = 0;  // bit t: target t accepts the node
     bool edge = false;
-    // A node that is accepted holds no target within its box unless it is as large as its
-    // distance: for theta <= 1 a target inside the box lies within sqrt(3) s / 2 + delta of
-    // the com, less than 0.93 of the acceptance radius, except for a node of size 0, where
-    // both are delta up to rounding. So the box is read only for acceptances at the edge.
-    const float lim = loose_theta ? INFINITY : H.x * 1.0001f;
+    // No target within a node's box accepts it. Such a target lies no farther from the com than
+    // the box's farthest corner, whose squared distance is in the record: a target's differences
+    // are at most the corner's, and rounding keeps that order through the same operations. So
+    // the box is read only where an accepted distance is not beyond it: for theta > 1, and for
+    // nodes a few ulps wide, whose com and centre are rounded onto the box's own bodies. (The
+    // quadrupole builds' records hold other radii; their rare fallback reads every box.)
+    const float lim = QUAD ? INFINITY : H.z;
     {
 #pragma clang fp contract(off)
 #pragma unroll
@@ -2094,8 +2097,8 @@ k_walk_target(const SegDesc* __restrict__ segs, const Tile* __restrict__ tiles, 
       if (__ballot(on) == 0ull) continue;
     }
     unsigned long long n_int = 0, n_vis = 0;
-    const Acc3 a = target_walk<KAHAN, COUNT>(s, k0, cnt, true, lane, words, masks, ~0u,
-                                               n_int, n_vis);
+    const Acc3 a = target_walk<KAHAN, COUNT, false>(s, k0, cnt, true, lane, words, masks, ~0u,
+                                                    n_int, n_vis);
     if (on) store_acc<false>(s, k, a, mode);
     if (COUNT) {
       n_int = wave_sum_u64(n_int);
@@ -2593,7 +2596,7 @@ __device__ __forceinline__ void drain_quads(Acc3& a, const WalkGroup& g, const f
 // Per-target fallback of a group whose stack would overflow: the aligned target sets of the
 // per-target walk that hold the group's bodies, so that a body's sum is the reference
 // build's bit for bit. The stack array serves as that walk's stack.
-template <bool KAHAN, bool COUNT>
+template <bool KAHAN, bool COUNT, bool QUAD>
 __device__ __forceinline__ Acc3 group_fallback(const SegDesc& s, const WalkGroup& g, uint32_t n,
                                                bool boxes, uint32_t lane, uint32_t* stk,
                                                unsigned long long& f_int,
@@ -2602,7 +2605,7 @@ __device__ __forceinline__ Acc3 group_fallback(const SegDesc& s, const WalkGroup
   for (uint32_t q = g.g0 / kTargets * kTargets; q < g.g0 + g.gcount; q += kTargets) {
     uint32_t mine = 0;  // the set's targets in this group (counted once)
     for (uint32_t i = 0; i < (uint32_t)kTargets; ++i) mine |= q + i - g.g0 < g.gcount ? 1u << i : 0u;
-    const Acc3 r = target_walk<KAHAN, COUNT>(
+    const Acc3 r = target_walk<KAHAN, COUNT, QUAD>(
         s, __builtin_amdgcn_readfirstlane(q), min(n - q, (uint32_t)kTargets), boxes, lane, stk,
         reinterpret_cast<uint8_t*>(stk + kOpenCap), mine, f_int, n_vis);
     const int src = (int)((g.k - q) & (kTargets - 1)) * kTargetLanes;
@@ -2724,7 +2727,7 @@ k_walk_group(const SegDesc* __restrict__ segs, const Tile* __restrict__ tiles, u
       if (overflow) {
         n_int = 0;
         n_quad = 0;
-        a = group_fallback<KAHAN, COUNT>(s, g, n, need_box, lane, stk, f_int, n_vis);
+        a = group_fallback<KAHAN, COUNT, QUAD>(s, g, n, need_box, lane, stk, f_int, n_vis);
         if (lane == 0) atomicAdd(&s.counters[kCntOverflow], 1ull);
       } else {  // the lists were drained in the last round
         fold_lanes<KAHAN>(a, g, lane);
@@ -2916,7 +2919,7 @@ k_walk_split(const SegDesc* __restrict__ segs, const Tile* __restrict__ tiles, u
       __syncthreads();
       if (last == 2u) {
         unsigned long long unused = 0;
-        a = group_fallback<KAHAN, false>(s, g, n, need_box, lane, stk, unused, unused);
+        a = group_fallback<KAHAN, false, QUAD>(s, g, n, need_box, lane, stk, unused, unused);
         if (lane == 0) atomicAdd(&s.counters[kCntOverflow], 1ull);
       } else {
         fold_lanes<KAHAN>(a, g, lane);
