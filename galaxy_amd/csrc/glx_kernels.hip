@@ -1884,6 +1884,45 @@ __device__ __forceinline__ void acc_add(Acc3& a, float tx, float ty, float tz) {
   }
 }
 
+// Two sums as one. Compensated, the rounding of each addition joins the compensations (the
+// exact error of a + b, D. Knuth's two-sum), so that nothing of the lanes' is lost.
+template <bool KAHAN>
+__device__ __forceinline__ void sum_join(float& v, float& c, float w, float d) {
+  const float t = v + w;
+  if (KAHAN) {
+    const float b = t - v;
+    c = (c + d) - ((v - (t - b)) + (w - b));
+  }
+  v = t;
+}
+template <bool KAHAN>
+__device__ __forceinline__ Acc3 acc_join(Acc3 a, const Acc3& b) {
+  sum_join<KAHAN>(a.x, a.cx, b.x, b.cx);
+  sum_join<KAHAN>(a.y, a.cy, b.y, b.cy);
+  sum_join<KAHAN>(a.z, a.cz, b.z, b.cz);
+  return a;
+}
+template <bool KAHAN>
+__device__ __forceinline__ Acc3 acc_shfl(const Acc3& a, int src) {
+  Acc3 r = {__shfl(a.x, src), __shfl(a.y, src), __shfl(a.z, src), 0.f, 0.f, 0.f};
+  if (KAHAN) {
+    r.cx = __shfl(a.cx, src);
+    r.cy = __shfl(a.cy, src);
+    r.cz = __shfl(a.cz, src);
+  }
+  return r;
+}
+template <bool KAHAN>
+__device__ __forceinline__ Acc3 acc_shfl_xor(const Acc3& a, int o) {
+  Acc3 r = {__shfl_xor(a.x, o), __shfl_xor(a.y, o), __shfl_xor(a.z, o), 0.f, 0.f, 0.f};
+  if (KAHAN) {
+    r.cx = __shfl_xor(a.cx, o);
+    r.cy = __shfl_xor(a.cy, o);
+    r.cz = __shfl_xor(a.cz, o);
+  }
+  return r;
+}
+
 template <bool KAHAN>
 __device__ __forceinline__ void store_acc(const SegDesc& s, uint32_t k, const Acc3& a, int mode) {
   const uint32_t n = s.n;
@@ -1915,7 +1954,7 @@ __device__ __forceinline__ void store_acc(const SegDesc& s, uint32_t k, const Ac
 // node against each of them (their positions are wave-uniform), adds the accepted ones'
 // monopole terms and the leaves' bodies to its own partial sums, and pushes the node's
 // children's word for the targets that open it. The partial sums are added over the wave
-// at the end. Every target accepts and opens exactly the nodes of the reference's
+// at the end, compensations included. Every target accepts and opens exactly the nodes of the reference's
 // pre-order walk (the distance test is written without contraction); only the order of
 // the sum differs.
 // Bound: one lane per target, each following its own chain of dependent node loads through
@@ -2042,33 +2081,20 @@ __device__ __forceinline__ Acc3 target_walk(const SegDesc& s, uint32_t k0, uint3
   }
   // Sum over the wave, halving the targets a lane holds with each of the first steps, so
   // that lanes [t kTargetLanes, (t + 1) kTargetLanes) end with target t's sum.
-  float vx[kTargets], vy[kTargets], vz[kTargets];
-#pragma unroll
-  for (int t = 0; t < kTargets; ++t) {
-    vx[t] = a[t].x - (KAHAN ? a[t].cx : 0.f);
-    vy[t] = a[t].y - (KAHAN ? a[t].cy : 0.f);
-    vz[t] = a[t].z - (KAHAN ? a[t].cz : 0.f);
-  }
   int o = 32;
 #pragma unroll
   for (int h = kTargets / 2; h > 0; h >>= 1, o >>= 1) {
     const bool up = (lane & (uint32_t)o) != 0u;
 #pragma unroll
     for (int t = 0; t < h; ++t) {
-      const float sx = up ? vx[t] : vx[t + h], sy = up ? vy[t] : vy[t + h],
-                  sz = up ? vz[t] : vz[t + h];
-      vx[t] = (up ? vx[t + h] : vx[t]) + __shfl_xor(sx, o);
-      vy[t] = (up ? vy[t + h] : vy[t]) + __shfl_xor(sy, o);
-      vz[t] = (up ? vz[t + h] : vz[t]) + __shfl_xor(sz, o);
+      const Acc3 give = up ? a[t] : a[t + h];
+      a[t] = acc_join<KAHAN>(up ? a[t + h] : a[t], acc_shfl_xor<KAHAN>(give, o));
     }
   }
 #pragma unroll
-  for (int w = kTargetLanes / 2; w > 0; w >>= 1) {
-    vx[0] += __shfl_xor(vx[0], w);
-    vy[0] += __shfl_xor(vy[0], w);
-    vz[0] += __shfl_xor(vz[0], w);
-  }
-  return {vx[0], vy[0], vz[0], 0.f, 0.f, 0.f};
+  for (int w = kTargetLanes / 2; w > 0; w >>= 1)
+    a[0] = acc_join<KAHAN>(a[0], acc_shfl_xor<KAHAN>(a[0], w));
+  return a[0];
 }
 
 // One wave per block and kTargets targets per wave; the tiles hold kBlock targets.
@@ -2099,7 +2125,7 @@ k_walk_target(const SegDesc* __restrict__ segs, const Tile* __restrict__ tiles, 
     unsigned long long n_int = 0, n_vis = 0;
     const Acc3 a = target_walk<KAHAN, COUNT, false>(s, k0, cnt, true, lane, words, masks, ~0u,
                                                     n_int, n_vis);
-    if (on) store_acc<false>(s, k, a, mode);
+    if (on) store_acc<KAHAN>(s, k, a, mode);
     if (COUNT) {
       n_int = wave_sum_u64(n_int);
       n_vis = wave_sum_u64(n_vis);
@@ -2609,8 +2635,8 @@ __device__ __forceinline__ Acc3 group_fallback(const SegDesc& s, const WalkGroup
         s, __builtin_amdgcn_readfirstlane(q), min(n - q, (uint32_t)kTargets), boxes, lane, stk,
         reinterpret_cast<uint8_t*>(stk + kOpenCap), mine, f_int, n_vis);
     const int src = (int)((g.k - q) & (kTargets - 1)) * kTargetLanes;
-    const float rx = __shfl(r.x, src), ry = __shfl(r.y, src), rz = __shfl(r.z, src);
-    if (g.owner && g.k - q < (uint32_t)kTargets) a = {rx, ry, rz, 0.f, 0.f, 0.f};
+    const Acc3 mine_sum = acc_shfl<KAHAN>(r, src);
+    if (g.owner && g.k - q < (uint32_t)kTargets) a = mine_sum;
     wave_lds_order();
   }
   return a;
