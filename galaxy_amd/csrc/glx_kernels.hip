@@ -3122,12 +3122,12 @@ __device__ __forceinline__ void sweep(PX sx, PM sm, uint32_t j0, uint32_t j1, F&
 }
 
 // Targets [64 blockIdx.x, +64) against the sources of chunk blockIdx.y, [c * len, min(n,
-// (c + 1) * len)), self excluded: by its zero distance where that gives a zero term (a
-// softening whose inverse cube is finite), else (SELF) by index. With one chunk the sums go
+// (c + 1) * len)), self excluded: by its zero distance where that gives a zero term (each of
+// the wave's own weights is finite: neither the mass nor the softening's inverse cube is
+// extreme), else by index, a compare and two selects a pair. With one chunk the sums go
 // straight to out (3 per target); with several, chunk c writes partial[(c * nt + t) * 3 +
 // axis] and k_direct_reduce adds the chunks in a fixed order, so results do not depend on
 // timing.
-template <bool SELF>
 __global__ void __launch_bounds__(64)
 k_direct_f64(const double* __restrict__ x, const double* __restrict__ m, uint32_t n,
              const uint32_t* __restrict__ targets, uint32_t nt, double g, double eps2,
@@ -3138,30 +3138,34 @@ k_direct_f64(const double* __restrict__ x, const double* __restrict__ m, uint32_
   double ax = 0.0, ay = 0.0, az = 0.0;
   const uint32_t j0 = blockIdx.y * chunk_len;
   const uint32_t j1 = (n - j0 < chunk_len) ? n : j0 + chunk_len;
-  sweep(cst(x), cst(m), j0, j1, [&](uint32_t j, const double* bx, const double* bm, auto count) {
-    constexpr int U = decltype(count)::value;
-    double dx[U], dy[U], dz[U], r2[U], w[U];
-    bool bad = false;
+  auto sum = [&](auto by_index) {
+    sweep(cst(x), cst(m), j0, j1, [&](uint32_t j, const double* bx, const double* bm, auto count) {
+      constexpr int U = decltype(count)::value;
+      double dx[U], dy[U], dz[U], r2[U], w[U];
+      bool bad = false;
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      dx[u] = bx[3 * u] - xi;
-      dy[u] = bx[3 * u + 1] - yi;
-      dz[u] = bx[3 * u + 2] - zi;
-      r2[u] = fma(dx[u], dx[u], fma(dy[u], dy[u], fma(dz[u], dz[u], eps2)));
-      w[u] = inv_cube(bm[u], r2[u], bad);
-    }
-    if (__builtin_expect(bad, 0)) {
+      for (int u = 0; u < U; ++u) {
+        dx[u] = bx[3 * u] - xi;
+        dy[u] = bx[3 * u + 1] - yi;
+        dz[u] = bx[3 * u + 2] - zi;
+        r2[u] = fma(dx[u], dx[u], fma(dy[u], dy[u], fma(dz[u], dz[u], eps2)));
+        w[u] = inv_cube(bm[u], r2[u], bad);
+      }
+      if (__builtin_expect(bad, 0)) {
 #pragma unroll
-      for (int u = 0; u < U; ++u) w[u] = inv_cube_ieee(bm[u], r2[u]);
-    }
+        for (int u = 0; u < U; ++u) w[u] = inv_cube_ieee(bm[u], r2[u]);
+      }
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const double q = (SELF && j + u == id) ? 0.0 : w[u];
-      ax = fma(dx[u], q, ax);
-      ay = fma(dy[u], q, ay);
-      az = fma(dz[u], q, az);
-    }
-  });
+      for (int u = 0; u < U; ++u) {
+        const double q = (decltype(by_index)::value && j + u == id) ? 0.0 : w[u];
+        ax = fma(dx[u], q, ax);
+        ay = fma(dy[u], q, ay);
+        az = fma(dz[u], q, az);
+      }
+    });
+  };
+  if (__ballot(!(fabs(inv_cube_ieee(m[id], eps2)) < 1e300)) == 0ull) sum(std::false_type{});
+  else sum(std::true_type{});
   if (t < nt) {
     double* o = out + ((size_t)blockIdx.y * nt + t) * 3;
     o[0] = g * ax;
@@ -3553,13 +3557,8 @@ hipError_t launch_direct_f64(hipStream_t st, const double* x, const double* m, u
   const bool whole = plan.chunks < 2u;
   const dim3 grid((nt + 63u) / 64u, whole ? 1u : plan.chunks), b(64);
   double* to = whole ? out : partial;
-  // eps^2 >= 1e-100: a body's term on itself is 0 times a finite number
-  if (eps2 >= 1e-100)
-    hipLaunchKernelGGL(k_direct_f64<false>, grid, b, 0, st, x, m, n, targets, nt, g, eps2,
-                       plan.chunk_len, to);
-  else
-    hipLaunchKernelGGL(k_direct_f64<true>, grid, b, 0, st, x, m, n, targets, nt, g, eps2,
-                       plan.chunk_len, to);
+  hipLaunchKernelGGL(k_direct_f64, grid, b, 0, st, x, m, n, targets, nt, g, eps2, plan.chunk_len,
+                     to);
   if (whole) return hipGetLastError();
   const uint32_t rblocks = (uint32_t)((3 * (size_t)nt + 63) / 64);
   hipLaunchKernelGGL(k_direct_reduce, dim3(rblocks), dim3(64 * kReduceWaves), 0, st, partial, nt,
