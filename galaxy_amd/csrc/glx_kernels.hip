@@ -3235,9 +3235,9 @@ k_potential_f64(const double* __restrict__ x, const double* __restrict__ m, uint
     }
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      // pairs j > i only (selected, not multiplied: the self pair may be infinite)
-      const double t = decltype(masked)::value && j + u <= row ? 0.0 : y[u];
-      pot = fma(bm[u], t, pot);
+      // pairs j > i only (selected, not multiplied: the self pair and the mass may be infinite)
+      const double t = fma(bm[u], y[u], pot);
+      pot = decltype(masked)::value && j + u <= row ? pot : t;
     }
   };
   sweep(cst(x), cst(m), j0, max(j0, diag_end),
@@ -3248,7 +3248,7 @@ k_potential_f64(const double* __restrict__ x, const double* __restrict__ m, uint
         [&](uint32_t j, const double* bx, const double* bm, auto count) {
           batch(j, bx, bm, count, std::false_type{});
         });
-  pot = row < n ? -g * m[row] * pot : 0.0;
+  pot = row < n && pot != 0.0 ? -g * m[row] * pot : 0.0;  // (0: no source of this chunk counts)
   pot = wave_sum(pot);
   if (threadIdx.x == 0) *o = pot;
 }

@@ -51,6 +51,17 @@ def test_own_mass_among_other_targets():
     assert not np.isfinite(np.delete(got, q, 0)).any()  # every other row holds the infinity
 
 
+@pytest.mark.parametrize("n", [2, 65, 200, 3000])
+@pytest.mark.parametrize("at", ["first", "inside"])
+def test_potential_with_an_infinite_mass(n, at):
+    """Only the pairs j > i count: an infinite mass makes the energy -inf, not NaN."""
+    rng = np.random.default_rng(n)
+    pos = rng.standard_normal((n, 3))
+    mass = rng.uniform(0.5, 1.5, n)
+    mass[0 if at == "first" else (n - 1) // 2] = np.inf
+    assert glx.Lbvh(1.0, 0.05, 0.5).potential_energy(pos, mass) == -np.inf
+
+
 # squared separations from below the smallest f32 to above the largest
 @pytest.mark.parametrize("scale", [1e-24, 1e-22, 1e-21, 3e-21, 1e-20, 3e-20, 1e-19, 1e-18,
                                    1e18, 1.5e19, 1e20])
