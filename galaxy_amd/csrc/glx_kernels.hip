@@ -2627,6 +2627,8 @@ __device__ __forceinline__ Acc3 group_fallback(const SegDesc& s, const WalkGroup
                                                bool boxes, uint32_t lane, uint32_t* stk,
                                                unsigned long long& f_int,
                                                unsigned long long& n_vis) {
+  // what depends on the lane is computed here, not kept in registers through every walk
+  if (!QUAD) asm volatile("" : "+v"(lane));
   Acc3 a = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   for (uint32_t q = g.g0 / kTargets * kTargets; q < g.g0 + g.gcount; q += kTargets) {
     uint32_t mine = 0;  // the set's targets in this group (counted once)
@@ -2662,10 +2664,14 @@ struct BoolTag {
 
 // The far-field build holds a 34-coefficient local expansion per lane: without a bound
 // the compiler takes about 147 VGPRs (3 waves per SIMD: walk +21%); at 4 waves per SIMD it
-// fits 128 VGPRs without spilling. The counting build is left unbounded (it only counts).
+// fits 128 VGPRs without spilling. The builds without quadrupoles are held to 80 VGPRs (6
+// waves per SIMD): the inlined per-target fallback took 84 (5 waves), 96 compensated. 2^22
+// bodies, theta = 0.5 / 1 / 1.3: 5,345 / 1,591 / 1,401 us at 5 waves, 5,289 / 1,514 / 1,315 at 6;
+// compensated 7,394 / 2,167 / 1,741 and 7,406 / 2,143 / 1,670. The counting build is left
+// unbounded (it only counts).
 template <bool KAHAN, bool COUNT, bool QUAD, bool FAR, bool WIDE>
 __global__ void __launch_bounds__(kGroup)
-__attribute__((amdgpu_waves_per_eu(COUNT ? 1 : 4)))
+__attribute__((amdgpu_waves_per_eu(COUNT ? 1 : (QUAD ? 4 : 6))))
 k_walk_group(const SegDesc* __restrict__ segs, const Tile* __restrict__ tiles, uint32_t ntiles,
              int mode) {
   __shared__ uint32_t stk[kStackCap];
