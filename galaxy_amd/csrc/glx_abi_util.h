@@ -176,12 +176,13 @@ inline void upload_state(const SegDesc& d, size_t n, const double* pos, const do
 }
 
 // One system's positions and velocities (either may be null) to the host.
-inline void download_state(const SegDesc& d, size_t n, double* pos, double* vel, hipStream_t st) {
+inline void download_state(const SegDesc& d, size_t n, double* pos, double* vel,
+                           const Batch& batch) {
   Copyout outs[2];
   int k = 0;
   if (pos) outs[k++] = Copyout{pos, d.x, 3 * n, false};
   if (vel) outs[k++] = Copyout{vel, d.v, 3 * n, true};
-  download(outs, k, st);
+  download(outs, k, batch);
 }
 
 // Phases of one resident KDK step, in launch order.

@@ -727,7 +727,7 @@ extern "C" int glx_sys_snapshot(glx_sys* s, double* pos, double* vel) {
   return guard([&] {
     if (!s) fail(GLX_EINVAL, "sys is NULL");
     if (s->n == 0) return;
-    download_state(s->seg.desc, s->n, pos, vel, s->st);
+    download_state(s->seg.desc, s->n, pos, vel, *s->batch);
   });
 }
 
@@ -737,7 +737,7 @@ extern "C" int glx_sys_snapshot_accel(glx_sys* s, double* acc) {
     const size_t n = s->n;
     if (n == 0) return;
     const Copyout out{acc, s->seg.desc.acc, 3 * n, true};
-    download(&out, 1, s->st);
+    download(&out, 1, *s->batch);
   });
 }
 
@@ -746,7 +746,7 @@ extern "C" int glx_sys_snapshot_mass(glx_sys* s, double* mass) {
     if (!s || !mass) fail(GLX_EINVAL, "NULL argument");
     if (s->n == 0) return;
     const Copyout out{mass, s->seg.desc.m, s->n, false};
-    download(&out, 1, s->st);
+    download(&out, 1, *s->batch);
   });
 }
 
@@ -813,11 +813,11 @@ extern "C" int glx_sys_run(glx_sys* s, const glx_run_config* cfg, const char* di
     std::vector<double> pos(3 * n), vel(3 * n), mass(n);
     if (n) {
       const Copyout out{mass.data(), s->seg.desc.m, n, false};
-      download(&out, 1, s->st);
+      download(&out, 1, *s->batch);
     }
     uint64_t emitted = 0;
     auto emit = [&](uint64_t step) {
-      if (n) download_state(s->seg.desc, n, pos.data(), vel.data(), s->st);
+      if (n) download_state(s->seg.desc, n, pos.data(), vel.data(), *s->batch);
       glx_snap_header h{};
       h.time = s->time;
       h.step = cfg->first_step + step;

@@ -303,7 +303,7 @@ extern "C" int glx_pool_job(glx_pool* p, uint64_t id, glx_job_info* out) {
 }
 
 static void job_snapshot(glx_pool* p, const Job* j, double* pos, double* vel) {
-  download_state(j->seg.desc, j->seg.desc.n, pos, vel, p->st);
+  download_state(j->seg.desc, j->seg.desc.n, pos, vel, *p->batch);
 }
 
 extern "C" int glx_pool_snapshot(glx_pool* p, uint64_t id, double* pos, double* vel) {
@@ -319,7 +319,7 @@ extern "C" int glx_pool_snapshot_accel(glx_pool* p, uint64_t id, double* acc) {
     const Job* j = find_job(p, id);
     pool_refresh(p);  // primes a job admitted since the last step
     const Copyout out{acc, j->seg.desc.acc, 3 * (size_t)j->seg.desc.n, true};
-    download(&out, 1, p->st);
+    download(&out, 1, *p->batch);
   });
 }
 
@@ -328,7 +328,7 @@ extern "C" int glx_pool_snapshot_mass(glx_pool* p, uint64_t id, double* mass) {
     if (!p || !mass) fail(GLX_EINVAL, "NULL argument");
     const Job* j = find_job(p, id);
     const Copyout out{mass, j->seg.desc.m, j->seg.desc.n, false};
-    download(&out, 1, p->st);
+    download(&out, 1, *p->batch);
   });
 }
 

@@ -37,8 +37,9 @@ struct Copyout {
   size_t count;
   bool widen;
 };
-// Waits for `st`, then copies every entry out; returns when all are written.
-void download(const Copyout* outs, int n, hipStream_t st);
+class Batch;
+// Waits for the batch's stream, then copies every entry out; returns when all are written.
+void download(const Copyout* outs, int n, const Batch& batch);
 
 // One system's device arrays (a single allocation carved into the arrays of
 // SegDesc). Capacity grows on demand and never shrinks.
@@ -104,6 +105,7 @@ class Batch {
   void diag(double* host_out /* nseg * kDiagRecord */);
 
   hipStream_t stream() const { return stream_; }
+  hipStream_t side() const { return side_; }  // idle whenever stream() is
 
  private:
   hipStream_t stream_;

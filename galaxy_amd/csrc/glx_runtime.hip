@@ -7,6 +7,7 @@
 #include <atomic>
 #include <condition_variable>
 #include <cstdlib>
+#include <memory>
 #include <mutex>
 #include <thread>
 
@@ -66,26 +67,28 @@ void ensure_device() {
 // link idle. Here pieces of 1 MiB go through pinned buffers, two per lane so that the next
 // piece is on the link while the last is written out, and large arrays are written by up to
 // four threads, which also share the page faults of a fresh destination. Positions and
-// velocities of 2^20 bodies into fresh memory: 7.5 -> 2.9 ms, of 2,000,003: 10.1 -> 3.7 ms.
+// velocities of 2^20 bodies into fresh memory: 7.4 -> 2.8 ms, of 2,000,003: 10.3 -> 4.0 ms.
+// The lanes are one pinned block, made once the downloads come to kLaneBytes and given back
+// with the last handle: making and freeing it takes about 0.3 ms, which a program that opens a
+// handle for one small snapshot would pay in full (two streams per lane and a block each, as
+// it was first done: 0.6 ms with one lane, 4.5 with four). Until then the copies are plain ones.
 // ----------------------------------------------------------------------------------
 
 namespace {
 constexpr size_t kPiece = (size_t)1 << 20;       // bytes on the link per piece
-constexpr size_t kLanes = 8;                     // lanes of the process, at most (16 MiB pinned)
+constexpr unsigned kLanes = 8;                   // lanes of the process (16 MiB pinned)
 constexpr size_t kPerThread = (size_t)4 << 20;   // device bytes worth another thread
 constexpr unsigned kDownloadThreads = 4;
+constexpr size_t kLaneBytes = (size_t)4 << 20;
 
-// A lane is used by one thread at a time; all are freed when the last Batch is gone.
-struct Lane {
-  unsigned char* buf[2] = {nullptr, nullptr};
-  hipStream_t st[2] = {nullptr, nullptr};
-};
-
+// A lane (two pieces of the block) is used by one thread at a time.
 struct LanePool {
   std::mutex mu;
   std::condition_variable back;
-  std::vector<Lane> free;
-  size_t made = 0, users = 0;
+  unsigned char* block = nullptr;
+  unsigned taken = 0;              // bit per lane
+  size_t plain = 0;                // bytes of plain downloads since a handle was first opened
+  size_t users = 0;
 };
 
 LanePool& lane_pool() {
@@ -93,83 +96,94 @@ LanePool& lane_pool() {
   return *p;
 }
 
-void lane_destroy(Lane& l) {
-  std::lock_guard<std::recursive_mutex> lock(device_memory_mutex());
-  for (int k = 0; k < 2; ++k) {
-    if (l.st[k]) (void)hipStreamDestroy(l.st[k]);
-    if (l.buf[k]) (void)hipHostFree(l.buf[k]);
-  }
-}
-
-hipError_t lane_make(Lane& l) {
-  std::lock_guard<std::recursive_mutex> lock(device_memory_mutex());
-  hipError_t e = hipSuccess;
-  for (int k = 0; k < 2 && e == hipSuccess; ++k) {
-    e = hipHostMalloc(reinterpret_cast<void**>(&l.buf[k]), kPiece, hipHostMallocDefault);
-    if (e == hipSuccess) e = hipStreamCreateWithFlags(&l.st[k], hipStreamNonBlocking);
-  }
-  if (e != hipSuccess) lane_destroy(l);
-  return e;
-}
-
-// A free lane, or a new one, or (at the limit) the next to come back.
-hipError_t lane_take(Lane& out) {
+// Index of a free lane for a download of `bytes`; with wait, the next to come back if all
+// are taken; -1: none.
+int lane_take(size_t bytes, bool wait) {
   LanePool& p = lane_pool();
   std::unique_lock<std::mutex> lock(p.mu);
-  for (;;) {
-    if (!p.free.empty()) {
-      out = p.free.back();
-      p.free.pop_back();
-      return hipSuccess;
+  if (!p.block) {
+    if (p.plain + bytes < kLaneBytes) {
+      p.plain += bytes;
+      return -1;
     }
-    if (p.made < kLanes) break;
+    std::lock_guard<std::recursive_mutex> device(device_memory_mutex());
+    if (hipHostMalloc(reinterpret_cast<void**>(&p.block), kLanes * 2 * kPiece,
+                      hipHostMallocDefault) != hipSuccess) {
+      p.block = nullptr;
+      fail(GLX_EDEVICE, "pinned memory for downloads");
+    }
+  }
+  for (;;) {
+    for (unsigned k = 0; k < kLanes; ++k)
+      if (!(p.taken >> k & 1u)) {
+        p.taken |= 1u << k;
+        return (int)k;
+      }
+    if (!wait) return -1;
     p.back.wait(lock);
   }
-  p.made += 1;
-  lock.unlock();
-  Lane l;
-  const hipError_t e = lane_make(l);
-  if (e != hipSuccess) {
-    lock.lock();
-    p.made -= 1;
-    p.back.notify_one();
-    return e;
-  }
-  out = l;
-  return hipSuccess;
 }
 
-void lane_give(const Lane& l) {
+void lane_give(int k) {
   LanePool& p = lane_pool();
   std::lock_guard<std::mutex> lock(p.mu);
-  p.free.push_back(l);  // (capacity kLanes is reserved with the first user)
+  p.taken &= ~(1u << k);
   p.back.notify_one();
 }
 
 void lanes_retain() {
   LanePool& p = lane_pool();
   std::lock_guard<std::mutex> lock(p.mu);
-  p.free.reserve(kLanes);
   p.users += 1;
 }
 
 void lanes_release() {
-  std::vector<Lane> gone;
-  {
-    LanePool& p = lane_pool();
-    std::lock_guard<std::mutex> lock(p.mu);
-    p.users -= 1;
-    if (p.users != 0) return;
-    gone.swap(p.free);
-    p.made -= gone.size();
-  }
-  for (Lane& l : gone) lane_destroy(l);
+  LanePool& p = lane_pool();
+  std::lock_guard<std::mutex> lock(p.mu);
+  p.users -= 1;
+  if (p.users != 0) return;
+  p.plain = 0;
+  if (!p.block) return;
+  std::lock_guard<std::recursive_mutex> device(device_memory_mutex());
+  (void)hipHostFree(p.block);
+  p.block = nullptr;
 }
 
-// Pieces of all arrays, taken in order from `next` by the threads of one download.
+// One thread's lane during a download. A thread that shares the streams with others waits for
+// its copies by events.
+struct Lane {
+  int index = -1;
+  unsigned char* buf[2] = {nullptr, nullptr};
+  hipEvent_t done[2] = {nullptr, nullptr};
+
+  bool open(size_t bytes, bool wait, bool shared) {
+    index = lane_take(bytes, wait);
+    if (index < 0) return false;
+    for (int k = 0; k < 2; ++k) {
+      buf[k] = lane_pool().block + (2 * (size_t)index + k) * kPiece;
+      if (shared && hipEventCreateWithFlags(&done[k], hipEventDisableTiming) != hipSuccess) {
+        done[k] = nullptr;
+        close();
+        return false;
+      }
+    }
+    return true;
+  }
+  void close() {
+    for (int k = 0; k < 2; ++k)
+      if (done[k]) (void)hipEventDestroy(done[k]);
+    done[0] = done[1] = nullptr;
+    if (index >= 0) lane_give(index);
+    index = -1;
+  }
+};
+
+// Pieces of all arrays, taken in order from `next` by the threads of one download. Their
+// copies go to the handle's two streams (one alone: no overlap for a few small pieces).
 struct Download {
   const Copyout* outs;
   int n;
+  hipStream_t st[2];
   std::atomic<size_t> next{0};
   std::atomic<int> error{hipSuccess};
 
@@ -194,13 +208,7 @@ struct Download {
     return false;
   }
 
-  void work() {
-    Lane lane;
-    hipError_t e = lane_take(lane);
-    if (e != hipSuccess) {
-      error = e;
-      return;
-    }
+  void work(const Lane& lane) {
     struct Held {
       const Copyout* o = nullptr;
       size_t first = 0, count = 0;
@@ -213,8 +221,9 @@ struct Download {
         return;
       }
       const size_t item = h.o->widen ? sizeof(float) : sizeof(double);
-      const hipError_t r = hipMemcpyAsync(lane.buf[k], static_cast<const char*>(h.o->src) + h.first * item,
-                                          h.count * item, hipMemcpyDeviceToHost, lane.st[k]);
+      hipError_t r = hipMemcpyAsync(lane.buf[k], static_cast<const char*>(h.o->src) + h.first * item,
+                                    h.count * item, hipMemcpyDeviceToHost, st[k]);
+      if (r == hipSuccess && lane.done[k]) r = hipEventRecord(lane.done[k], st[k]);
       if (r != hipSuccess) {
         error = r;
         h.o = nullptr;
@@ -223,7 +232,8 @@ struct Download {
     start(0);
     for (int k = 0; held[k].o; k ^= 1) {
       start(k ^ 1);
-      const hipError_t r = hipStreamSynchronize(lane.st[k]);
+      const hipError_t r =
+          lane.done[k] ? hipEventSynchronize(lane.done[k]) : hipStreamSynchronize(st[k]);
       if (r != hipSuccess) {
         error = r;
         break;
@@ -237,16 +247,36 @@ struct Download {
         memcpy(dst, lane.buf[k], h.count * sizeof(double));
       }
     }
-    if (error != hipSuccess)  // nothing of this lane stays in flight
-      for (int k = 0; k < 2; ++k) (void)hipStreamSynchronize(lane.st[k]);
-    lane_give(lane);
+    if (error != hipSuccess)  // nothing stays in flight to the lane
+      for (int k = 0; k < 2; ++k) (void)hipStreamSynchronize(st[k]);
   }
 };
+
+// The same without lanes: whole arrays, f32 through a buffer of their own.
+void download_plain(const Copyout* outs, int n, hipStream_t st) {
+  std::vector<std::unique_ptr<float[]>> narrow(n);
+  for (int i = 0; i < n; ++i)
+    if (outs[i].widen) narrow[i].reset(new float[outs[i].count]);
+  hipError_t r = hipSuccess;
+  for (int i = 0; i < n && r == hipSuccess; ++i) {
+    const Copyout& o = outs[i];
+    r = hipMemcpyAsync(o.widen ? (void*)narrow[i].get() : (void*)o.dst, o.src,
+                       o.count * (o.widen ? sizeof(float) : sizeof(double)), hipMemcpyDeviceToHost,
+                       st);
+  }
+  const hipError_t w = hipStreamSynchronize(st);
+  check(r != hipSuccess ? r : w, "download");
+  for (int i = 0; i < n; ++i)
+    if (outs[i].widen)
+      for (size_t q = 0; q < outs[i].count; ++q) outs[i].dst[q] = (double)narrow[i][q];
+}
+
 }  // namespace
 
-void download(const Copyout* outs, int n, hipStream_t st) {
+void download(const Copyout* outs, int n, const Batch& batch) {
+  const hipStream_t st = batch.stream();
   check(hipStreamSynchronize(st), "hipStreamSynchronize");
-  Download d{outs, n};
+  Download d{outs, n, {st, batch.side()}};
   size_t bytes = 0;
   for (int i = 0; i < n; ++i) bytes += outs[i].count * (outs[i].widen ? sizeof(float) : sizeof(double));
   if (bytes == 0) return;
@@ -254,18 +284,26 @@ void download(const Copyout* outs, int n, hipStream_t st) {
   const size_t pieces = d.pieces();
   if (threads > pieces) threads = pieces;
   if (threads > kDownloadThreads) threads = kDownloadThreads;
+  Lane mine;
+  if (!mine.open(bytes, true, threads > 1)) return download_plain(outs, n, st);
   std::thread more[kDownloadThreads];
   size_t started = 0;
   for (size_t t = 1; t < threads; ++t) {
     try {
-      more[started] = std::thread([&d] { d.work(); });
+      more[started] = std::thread([&d, bytes] {
+        Lane lane;
+        if (!lane.open(bytes, false, true)) return;  // the others take its pieces
+        d.work(lane);
+        lane.close();
+      });
     } catch (...) {
-      break;  // no thread to be had: the others take its pieces
+      break;  // no thread to be had: the same
     }
     ++started;
   }
-  d.work();
+  d.work(mine);
   for (size_t t = 0; t < started; ++t) more[t].join();
+  mine.close();
   check((hipError_t)d.error.load(), "download");
 }
 
