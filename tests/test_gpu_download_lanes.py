@@ -1,6 +1,6 @@
 """Downloads when pinned lanes run short: more threads than the process has lanes (each waits
-its turn); and the lanes of one handle after another. Every download returns what was
-uploaded."""
+its turn), and none to be had at all (GLX_DOWNLOAD_LANES=0 caps them), where snapshots come
+through plain copies instead. Every download returns what was uploaded."""
 from __future__ import annotations
 
 import threading
@@ -9,6 +9,7 @@ import numpy as np
 import pytest
 
 import galaxy_amd as glx
+from galaxy_amd.pool import Pool
 
 pytestmark = pytest.mark.gpu
 
@@ -57,6 +58,29 @@ def test_more_threads_than_lanes():
     assert not errs, errs
     assert not any(t.is_alive() for t in ts)
     assert sorted(done) == list(range(count))
+
+
+@pytest.mark.parametrize("lanes", ["0", "1", "2"])
+@pytest.mark.parametrize("n", [1, 43_691, 87_382, 470_001])
+def test_few_or_no_lanes(monkeypatch, lanes, n):
+    monkeypatch.setenv("GLX_DOWNLOAD_LANES", lanes)
+    want = state(n, n)
+    r = glx.GpuResidentLeapfrog(1.0, 0.05, 0.5)
+    r.upload(*want)
+    check(resident(r), want)
+    r.step(1e-3)  # a later kernel launch reports no error left behind
+    acc = r.snapshot_accel()
+    r.close()
+    p = Pool(1 << 30)
+    job = p.admit(*want, softening=0.05, theta=0.5, dt=1e-3)
+    check((*p.snapshot(job), p.snapshot_mass(job)), want)
+    p.close()
+    monkeypatch.delenv("GLX_DOWNLOAD_LANES")
+    r = glx.GpuResidentLeapfrog(1.0, 0.05, 0.5)
+    r.upload(*want)
+    r.step(1e-3)
+    assert np.array_equal(r.snapshot_accel(), acc)
+    r.close()
 
 
 def test_handles_one_after_the_other():
