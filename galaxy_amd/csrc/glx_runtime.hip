@@ -82,7 +82,8 @@ constexpr size_t kPerThread = (size_t)4 << 20;   // device bytes worth another t
 constexpr unsigned kDownloadThreads = 4;
 constexpr size_t kLaneBytes = (size_t)4 << 20;
 
-// A lane (two pieces of the block) is used by one thread at a time.
+// A lane (two pieces of the block) is used by one thread at a time. The block is portable
+// memory: any device's copies may use it.
 struct LanePool {
   std::mutex mu;
   std::condition_variable back;
@@ -119,7 +120,7 @@ int lane_take(size_t bytes, bool wait) {
     }
     std::lock_guard<std::recursive_mutex> device(device_memory_mutex());
     if (hipHostMalloc(reinterpret_cast<void**>(&p.block), kLanes * 2 * kPiece,
-                      hipHostMallocDefault) != hipSuccess) {
+                      hipHostMallocPortable) != hipSuccess) {
       (void)hipGetLastError();  // the plain copies take over: nothing for a later call to find
       p.block = nullptr;
       return -1;
@@ -162,7 +163,8 @@ void lanes_release() {
 }
 
 // One thread's lane during a download. A thread that shares the streams with others waits for
-// its copies by events.
+// its copies by events; those belong to the device that is current when the lane is opened,
+// which is the streams'.
 struct Lane {
   int index = -1;
   unsigned char* buf[2] = {nullptr, nullptr};
@@ -284,6 +286,20 @@ void download_plain(const Copyout* outs, int n, hipStream_t st) {
       for (size_t q = 0; q < outs[i].count; ++q) outs[i].dst[q] = (double)narrow[i][q];
 }
 
+// Makes a device current for a scope.
+struct OnDevice {
+  int was = -1;
+  explicit OnDevice(int device) {
+    int now = 0;
+    check(hipGetDevice(&now), "hipGetDevice");
+    if (now == device) return;
+    check(hipSetDevice(device), "hipSetDevice");
+    was = now;
+  }
+  ~OnDevice() {
+    if (was >= 0) (void)hipSetDevice(was);
+  }
+};
 }  // namespace
 
 void download(const Copyout* outs, int n, const Batch& batch) {
@@ -293,6 +309,9 @@ void download(const Copyout* outs, int n, const Batch& batch) {
   size_t bytes = 0;
   for (int i = 0; i < n; ++i) bytes += outs[i].count * (outs[i].widen ? sizeof(float) : sizeof(double));
   if (bytes == 0) return;
+  hipDevice_t device = 0;  // the handle's, whatever is current in this thread; new threads start at 0
+  check(hipStreamGetDevice(st, &device), "hipStreamGetDevice");
+  OnDevice on(device);
   size_t threads = bytes / kPerThread;
   const size_t pieces = d.pieces();
   if (threads > pieces) threads = pieces;
@@ -303,9 +322,10 @@ void download(const Copyout* outs, int n, const Batch& batch) {
   size_t started = 0;
   for (size_t t = 1; t < threads; ++t) {
     try {
-      more[started] = std::thread([&d, bytes] {
+      more[started] = std::thread([&d, bytes, device] {
         Lane lane;
-        if (!lane.open(bytes, false, true)) return;  // the others take its pieces
+        if (hipSetDevice(device) != hipSuccess || !lane.open(bytes, false, true))
+          return;  // the others take its pieces
         d.work(lane);
         lane.close();
       });
