@@ -58,8 +58,9 @@ struct __align__(16) Node {
   float4 a;  // centre of mass (origin-relative f32), mass
   float4 h;  // squared acceptance radius (s/theta + delta)^2, children as walk entries
              // (enc_entries, as bits); then, with quadrupoles, the group walk's squared
-             // monopole-band radius and the node's radius about its com, otherwise the
-             // squared distance from the com to the box's farthest corner
+             // monopole-band radius and the node's radius about its com (negative: a point),
+             // otherwise the squared distance from the com to the box's farthest corner and
+             // the node's size
 };
 struct __align__(16) NodeBox {
   float4 lo;  // AABB min (origin-relative f32), first leaf (as bits)

@@ -1334,13 +1334,15 @@ __device__ __forceinline__ void store_node(const SegDesc& s, uint32_t j, const A
   if (QUAD) {
     // the group walk's classifier radii: squared monopole-band radius (s / (theta
     // mono_ratio) + delta; FLT_MAX when the band is off) and the node's radius about its
-    // com (far-field test)
+    // com (far-field test), negative for a node that is a single point
     const float rn = sqrtf(fmaf(ex, ex, fmaf(ey, ey, ez * ez)));
     const float rm = fmaf(size, s.mono_inv, delta);
-    nd.h = make_float4(rcrit * rcrit, ch, s.mono_inv > 0.f ? rm * rm : 3.4e38f, rn);
+    nd.h = make_float4(rcrit * rcrit, ch, s.mono_inv > 0.f ? rm * rm : 3.4e38f,
+                       size > 0.f ? rn : -rn);
   } else {
-    nd.h = make_float4(rcrit * rcrit, ch, ex * ex + ey * ey + ez * ez, 0.f);
+    nd.h = make_float4(rcrit * rcrit, ch, ex * ex + ey * ey + ez * ez, size);
   }
+  if (!(rcrit >= 0.0f)) nd.h.x = nd.h.w = INFINITY;  // a NaN com: nobody accepts it
   const size_t j2 = 2 * (size_t)j;
   gstore4(reinterpret_cast<float4*>(s.node), j2, nd.a);
   gstore4(reinterpret_cast<float4*>(s.node), j2 + 1, nd.h);
@@ -1965,6 +1967,13 @@ __device__ __forceinline__ void store_acc(const SegDesc& s, uint32_t k, const Ac
 // each node load between 4 targets measured best over that range (2 targets: 20, 64 us,
 // 15 ms; 8: 32, 74 us, 10.7 ms). 64 VGPRs (8 waves per SIMD; the compiler takes 67
 // unasked) are worth 4% at 100,003 bodies.
+// Squared distance from a node's com to its box's farthest corner, from the second part of its
+// record; not less than any target's in the box.
+template <bool QUAD>
+__device__ __forceinline__ float corner_distance2(const float4& H) {
+  return QUAD ? H.w * H.w * 1.000002f : H.z;
+}
+
 constexpr int kTargets = 4;
 constexpr int kTargetLanes = 64 / kTargets;  // lanes that end with one target's sum
 // Stack entries (children word of an opened node, mask of the targets that opened it).
@@ -2009,8 +2018,10 @@ __device__ __forceinline__ Acc3 target_walk(const SegDesc& s, uint32_t k0, uint3
     // are at most the corner's, and rounding keeps that order through the same operations. So
     // the box is read only where an accepted distance is not beyond it: for theta > 1, and for
     // nodes a few ulps wide, whose com and centre are rounded onto the box's own bodies. (The
-    // quadrupole builds' records hold other radii; their rare fallback reads every box.)
-    const float lim = QUAD ? INFINITY : H.z;
+    // quadrupole builds' records hold other radii; their rare fallback reads every box.) Without
+    // boxes, in the group walk's fallback, nothing that near is accepted, a point excepted.
+    const float corner2 = corner_distance2<QUAD>(H);
+    const float lim = QUAD ? INFINITY : corner2;
     {
 #pragma clang fp contract(off)
 #pragma unroll
@@ -2033,6 +2044,11 @@ __device__ __forceinline__ Acc3 target_walk(const SegDesc& s, uint32_t k0, uint3
         if ((B.x <= mx[t]) & (mx[t] <= C.x) & (B.y <= my[t]) & (my[t] <= C.y) &
             (B.z <= mz[t]) & (mz[t] <= C.z))
           acc &= ~(1u << t);
+    }
+    if (!boxes) {
+#pragma unroll
+      for (int t = 0; t < kTargets; ++t)
+        if (H.w > 0.0f && d2[t] <= corner2) acc &= ~(1u << t);
     }
     const uint32_t live = massive ? mk : 0u;
     const uint32_t self = u - k0 < (uint32_t)kTargets ? 1u << (u - k0) : 0u;
@@ -2383,6 +2399,7 @@ struct WalkGroup {
   bool owner, valid;
   float4 me;
   float gx0, gy0, gz0, gx1, gy1, gz1, cx, cy, cz, hx, hy, hz, rg;
+  float near2;  // squared distance within which no node is accepted (theta <= 1), points excepted
 };
 
 template <bool FAR>
@@ -2422,6 +2439,15 @@ __device__ __forceinline__ void walk_group_box(const SegDesc& s, WalkGroup& g) {
   g.hx = 0.5f * (g.gx1 - g.gx0);
   g.hy = 0.5f * (g.gy1 - g.gy0);
   g.hz = 0.5f * (g.gz1 - g.gz0);
+  // Distances from the box come from its centre and half extent, each rounded to 2^-24 of its
+  // coordinates, so they may be 7 of these too large: a node much smaller than that at the box's
+  // edge would be accepted by the group that holds its bodies. For theta <= 1 that takes a com
+  // within 2^-24 * 131 of the coordinates (theta = 1: s (1 - sqrt(3) / 2) below 8.7 of these,
+  // the radius below 124); nothing within 2^-15 is accepted.
+  const float most = fmaxf(fmaxf(fmaxf(-g.gx0, g.gx1), fmaxf(-g.gy0, g.gy1)),
+                           fmaxf(-g.gz0, g.gz1));
+  const float t = most * 0x1p-15f;
+  g.near2 = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(fmaxf(t * t, 1.2e-38f))));
   g.rg = FAR ? sqrtf(fmaf(g.hx, g.hx, fmaf(g.hy, g.hy, g.hz * g.hz))) : 0.0f;
 }
 
@@ -2501,8 +2527,8 @@ __device__ __forceinline__ bool walk_round(const SegDesc& s, const WalkSeg& w, c
     // Every point of the node's box lies within sqrt(3) s / 2 + delta of its com
     // (half its diagonal from the box centre, delta from there to the com), and an
     // accepted com is at least s / theta + delta from the group box, so for theta <= 1
-    // (1 / theta > sqrt(3) / 2 with a margin) acceptance implies disjoint boxes. (A
-    // node of size 0 is one point, whose monopole is exact for every body.)
+    // (1 / theta > sqrt(3) / 2 with a margin) acceptance implies disjoint boxes, beyond
+    // near2. (A node of size 0 is one point, whose monopole is exact for every body.)
     if (w.loose_theta)
       apart = (Cc.x < g.gx0) | (B.x > g.gx1) | (Cc.y < g.gy0) | (B.y > g.gy1) |
               (Cc.z < g.gz0) | (B.z > g.gz1);
@@ -2517,7 +2543,10 @@ __device__ __forceinline__ bool walk_round(const SegDesc& s, const WalkSeg& w, c
   const float dmin2 = ex * ex + ey * ey + ez * ez;
   const bool massive = A.w > 0.0f;
   const bool node_live = is_node & massive;
-  const bool accept = node_live & apart & (dmin2 >= H.x);  // boxes disjoint too
+  // the acceptance radius, at least near2 for a node that is not a single point (one
+  // instruction more: H.w > 0 there); above theta = 1 the boxes have been compared
+  const float lim = BOX && w.loose_theta ? H.x : __builtin_amdgcn_fmed3f(H.x, g.near2, H.w * 1e30f);
+  const bool accept = node_live & apart & (dmin2 >= lim);  // boxes disjoint too
   const bool near = node_live & !accept;
   const bool bkt = BOX & near & (ncount <= w.bucket);  // (leaf_size > 1 needs boxes)
   const bool open = near & !bkt;
@@ -2525,7 +2554,7 @@ __device__ __forceinline__ bool walk_round(const SegDesc& s, const WalkSeg& w, c
   // about its com from the record)
   bool far = false;
   if (FAR) {
-    const float rn = H.w + g.rg;
+    const float rn = fabsf(H.w) + g.rg;
     far = accept & (rn * rn <= s.far2 * fmaf(dx, dx, fmaf(dy, dy, dz * dz)));
   }
   // an accepted node that also passes the opening test at theta * mono_ratio is a
@@ -2621,7 +2650,8 @@ __device__ __forceinline__ void drain_quads(Acc3& a, const WalkGroup& g, const f
 
 // Per-target fallback of a group whose stack would overflow: the aligned target sets of the
 // per-target walk that hold the group's bodies, so that a body's sum is the reference
-// build's bit for bit. The stack array serves as that walk's stack.
+// build's bit for bit (but for nodes a few ulps wide, opened there without their boxes). The
+// stack array serves as that walk's stack.
 template <bool KAHAN, bool COUNT, bool QUAD>
 __device__ __forceinline__ Acc3 group_fallback(const SegDesc& s, const WalkGroup& g, uint32_t n,
                                                bool boxes, uint32_t lane, uint32_t* stk,
@@ -2667,11 +2697,11 @@ struct BoolTag {
 // fits 128 VGPRs without spilling. The builds without quadrupoles are held to 80 VGPRs (6
 // waves per SIMD): the inlined per-target fallback took 84 (5 waves), 96 compensated. 2^22
 // bodies, theta = 0.5 / 1 / 1.3: 5,345 / 1,591 / 1,401 us at 5 waves, 5,289 / 1,514 / 1,315 at 6;
-// compensated 7,394 / 2,167 / 1,741 and 7,406 / 2,143 / 1,670. The counting build is left
-// unbounded (it only counts).
+// compensated 7,394 / 2,167 / 1,741 and 7,406 / 2,143 / 1,670. Those with quadrupoles and no
+// far field fit 96 VGPRs (5 waves). The counting build is left unbounded (it only counts).
 template <bool KAHAN, bool COUNT, bool QUAD, bool FAR, bool WIDE>
 __global__ void __launch_bounds__(kGroup)
-__attribute__((amdgpu_waves_per_eu(COUNT ? 1 : (QUAD ? 4 : 6))))
+__attribute__((amdgpu_waves_per_eu(COUNT ? 1 : (QUAD ? (FAR ? 4 : 5) : 6))))
 k_walk_group(const SegDesc* __restrict__ segs, const Tile* __restrict__ tiles, uint32_t ntiles,
              int mode) {
   __shared__ uint32_t stk[kStackCap];
