@@ -95,6 +95,16 @@ inline void validate_direct(size_t n, const double* pos, const double* mass,
     if (targets[t] >= n) fail(GLX_EINVAL, "target index out of range");
 }
 
+// The group walk's distance of a com from a group box may come out 4 sqrt(3) c too large, c being
+// 2^-24 of the box's coordinates (centre, half extent and their differences rounded); a node's
+// centre may be sqrt(3) c off. So for theta <= 1 a node of size s that holds one of the group's
+// bodies is accepted at most where s (1 / theta - sqrt(3) / 2) <= 8.7 c, at a distance of at
+// most sqrt(3) s + 17 c (its com up to 8 c out of its box). This is a third more, as a share of
+// the coordinates: 173 c at theta = 1, 42 c at 0.5. Above theta = 1 the boxes are compared.
+inline float near_share(double theta) {
+  return (float)theta > 1.0f ? 0.0f : (float)((24.0 + 20.0 * theta / (1.0 - 0.866 * theta)) * 0x1p-24);
+}
+
 inline void fill_params(SegDesc& d, const glx_params& p, uint32_t n) {
   d.n = n;
   d.g = (float)p.g;
@@ -105,6 +115,7 @@ inline void fill_params(SegDesc& d, const glx_params& p, uint32_t n) {
   d.group_size = p.group_size ? p.group_size : (uint32_t)kGroup;
   d.group_lanes = p.group_lanes ? p.group_lanes : 4u;
   d.far2 = (float)(p.far_theta * p.far_theta);
+  d.near_coord = near_share(p.theta);
   d.mono_inv = p.mono_ratio > 0.0 ? (float)(1.0 / (p.theta * p.mono_ratio)) : 0.0f;
 }
 

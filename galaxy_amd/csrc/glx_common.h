@@ -185,6 +185,7 @@ struct SegDesc {
   uint32_t stack_cap;   // group walk: stack entries before the per-target fallback (0: all)
   float g, eps2, theta, half_dt;
   float far2;  // squared far-field ratio: (node radius + group radius)^2 <= far2 * R^2
+  float near_coord;  // near_share(theta): the group walk's least distance, per coordinate
   float mono_inv;  // 1 / (theta mono_ratio): accepted nodes this far are monopoles (0: off)
   double dt;
 };

@@ -2441,12 +2441,11 @@ __device__ __forceinline__ void walk_group_box(const SegDesc& s, WalkGroup& g) {
   g.hz = 0.5f * (g.gz1 - g.gz0);
   // Distances from the box come from its centre and half extent, each rounded to 2^-24 of its
   // coordinates, so they may be 7 of these too large: a node much smaller than that at the box's
-  // edge would be accepted by the group that holds its bodies. For theta <= 1 that takes a com
-  // within 2^-24 * 131 of the coordinates (theta = 1: s (1 - sqrt(3) / 2) below 8.7 of these,
-  // the radius below 124); nothing within 2^-15 is accepted.
+  // edge would be accepted by the group that holds its bodies. Nothing within near_coord of the
+  // coordinates is accepted, which is farther than any such node (near_share).
   const float most = fmaxf(fmaxf(fmaxf(-g.gx0, g.gx1), fmaxf(-g.gy0, g.gy1)),
                            fmaxf(-g.gz0, g.gz1));
-  const float t = most * 0x1p-15f;
+  const float t = most * s.near_coord;
   g.near2 = __uint_as_float(__builtin_amdgcn_readfirstlane(__float_as_uint(fmaxf(t * t, 1.2e-38f))));
   g.rg = FAR ? sqrtf(fmaf(g.hx, g.hx, fmaf(g.hy, g.hy, g.hz * g.hz))) : 0.0f;
 }

@@ -1,5 +1,5 @@
 """The group walk's acceptance for theta <= 1 (galaxy_amd/csrc/glx_kernels.hip, walk_group_box and
-walk_round) on its f32 arithmetic, for nodes down to an ulp wide at the edge of group boxes up
+walk_round, near_share) on its f32 arithmetic, for nodes down to an ulp wide at the edge of group boxes up
 to 1e6 times larger: a node that holds a body within the group box is never accepted, unless
 it is a single point. The acceptance radius alone would let many through."""
 from __future__ import annotations
@@ -32,7 +32,7 @@ def cases(rng, n):
 def test_no_node_with_a_body_in_the_group_is_accepted():
     rng = np.random.default_rng(4)
     by_radius = 0
-    for theta in (0.3, 0.5, 0.7, 0.9, 1.0):
+    for theta in (0.05, 0.3, 0.5, 0.7, 0.9, 1.0):
         for _ in range(4):
             lo, hi, mn, mx, com = cases(rng, 100_000)
             cen, half = ((mn + mx) * f(0.5)).astype(f), ((mx - mn) * f(0.5)).astype(f)
@@ -45,6 +45,7 @@ def test_no_node_with_a_body_in_the_group_is_accepted():
             accept = (dmin2 >= (r * r).astype(f)) & (size > 0)
             by_radius += int(accept.sum())
             most = np.maximum(np.abs(lo), np.abs(hi)).max(axis=1)
-            t = (most * f(2.0 ** -15)).astype(f)
+            share = f((24 + 20 * theta / (1 - 0.866 * theta)) * 2.0 ** -24)
+            t = (most * share).astype(f)
             assert not (accept & (dmin2 >= t * t)).any(), theta
     assert by_radius > 10_000
