@@ -636,11 +636,11 @@ k_radix_downsweep(const SegDesc* __restrict__ segs, const Tile* __restrict__ til
 // 3b. the same sort for launches of few bodies: buckets by sampled splitters, then every
 //     bucket sorted in one block's LDS. The digit passes above are bound there by their
 //     launches, three a pass (63-bit keys, 2,000 bodies: 24 launches, 109 us; 30-bit keys,
-//     16,384 bodies: 9 launches, 57 us). Here a system of up to kLocalDirect bodies takes one
-//     launch and a larger one four, whatever the key width: 23 us, and 39 us in all; 63-bit
-//     keys, 100,003 bodies: 127 -> 69 us. The digits that no two keys of a bucket differ in
-//     are left out. Equal keys keep index order: splitters
-//     compare (key, index), and every scatter is stable.
+//     16,384 bodies, 10-bit digits: 9 launches, 48 us). Here a system of up to kLocalDirect
+//     bodies takes one launch and a larger one four, whatever the key width: 23 us, and 38 us
+//     in all; 63-bit keys, 100,003 bodies: 127 -> 69 us. The digits that no two keys of a
+//     bucket differ in are left out. Equal keys keep index order: splitters compare (key,
+//     index), and every scatter is stable.
 // ----------------------------------------------------------------------------------
 
 constexpr int kLocalThreads = 1024, kLocalItems = 6;
@@ -1950,23 +1950,6 @@ __device__ __forceinline__ void store_acc(const SegDesc& s, uint32_t k, const Ac
   }
 }
 
-// Per-target walk (the reference's criterion for every target, solvers/src/lbvh.rs:469-524):
-// one wave walks for kTargets Morton-consecutive targets, 64 nodes at a time, one per lane.
-// A node carries the mask of the targets that opened all its ancestors; a lane tests its
-// node against each of them (their positions are wave-uniform), adds the accepted ones'
-// monopole terms and the leaves' bodies to its own partial sums, and pushes the node's
-// children's word for the targets that open it. The partial sums are added over the wave
-// at the end, compensations included. Every target accepts and opens exactly the nodes of the reference's
-// pre-order walk (the distance test is written without contraction); only the order of
-// the sum differs.
-// Bound: one lane per target, each following its own chain of dependent node loads through
-// the pre-order, took 649 us for 1,000 bodies (16 waves on the chip), 1,757 us for a
-// 16,384-body Plummer sphere and 130 ms for a 2^18-body collision. With 64 nodes per step
-// the chain is the tree's depth and the wave's loads are in flight together: 23, 56 us and
-// 8.7 ms, now bound by the node gathers and about 140 VALU instructions a round. Sharing
-// each node load between 4 targets measured best over that range (2 targets: 20, 64 us,
-// 15 ms; 8: 32, 74 us, 10.7 ms). 64 VGPRs (8 waves per SIMD; the compiler takes 67
-// unasked) are worth 4% at 100,003 bodies.
 // Squared distance from a node's com to its box's farthest corner, from the second part of its
 // record; not less than any target's in the box.
 template <bool QUAD>
@@ -1974,6 +1957,23 @@ __device__ __forceinline__ float corner_distance2(const float4& H) {
   return QUAD ? H.w * H.w * 1.000002f : H.z;
 }
 
+// Per-target walk (the reference's criterion for every target, solvers/src/lbvh.rs:469-524):
+// one wave walks for kTargets Morton-consecutive targets, 64 nodes at a time, one per lane.
+// A node carries the mask of the targets that opened all its ancestors; a lane tests its
+// node against each of them (their positions are wave-uniform), adds the accepted ones'
+// monopole terms and the leaves' bodies to its own partial sums, and pushes the node's
+// children's word for the targets that open it. The partial sums are added over the wave
+// at the end, compensations included. Every target accepts and opens exactly the nodes of the
+// reference's pre-order walk (the distance test is written without contraction, and the box
+// is read wherever a target inside it could pass it); only the order of the sum differs.
+// Bound: one lane per target, each following its own chain of dependent node loads through
+// the pre-order, took 605 to 649 us for 1,000 bodies (16 waves on the chip), 1,782 us for a
+// 16,384-body Plummer sphere and 177 ms for a 2^18-body collision. With 64 nodes per step
+// the chain is the tree's depth and the wave's loads are in flight together: 23, 55 us and
+// 9.4 ms (2,621 -> 231 us at 100,003 bodies), now bound by the node gathers and about 140 VALU
+// instructions a round. Sharing each node load between 4 targets measured best over that
+// range (2 targets: 20, 64 us, 15 ms; 8: 32, 74 us, 10.7 ms). 64 VGPRs are 8 waves per SIMD,
+// worth 4% at 100,003 bodies.
 constexpr int kTargets = 4;
 constexpr int kTargetLanes = 64 / kTargets;  // lanes that end with one target's sum
 // Stack entries (children word of an opened node, mask of the targets that opened it).
